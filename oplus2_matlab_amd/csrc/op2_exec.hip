@@ -1436,7 +1436,8 @@ bool known_zero(op_dat d) {
 }
 
 // During a capture: the dats of a save_soln (q, qold) that still hold the
-// same values.
+// same values.  Every launch that writes either ends that: note_writes, and
+// flush_chain for the stages.
 std::pair<op_dat, op_dat> &copied_dats() {
   static std::pair<op_dat, op_dat> p;
   return p;
@@ -3046,6 +3047,11 @@ void flush_chain() {
   c.swap(chain());
   if (c.empty()) return;
   const CellTiles *march = march_tiles(c);
+  // the stages write q: it equals qold again only where the last one took in
+  // a save_soln
+  const Stage &end = c.back();
+  copied_dats() = end.save.empty() ? std::pair<op_dat, op_dat>{}
+                                   : std::make_pair(end.save[0].dat, end.save[1].dat);
   if (march) {
     if (c[0].rb == 8)
       run_march<double>(c, march);
