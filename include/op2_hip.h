@@ -110,7 +110,9 @@ op_dat op2_decl_dat_char(op_set set, int dim, char const *type, int size,
                          char *data, char const *name);
 
 /* op_decl_const_char, airfoil/airfoil_kernels.cu:50-53: stores a named
- * constant (dim elements of size bytes) for the device loops */
+ * constant (dim elements of size bytes) for the device loops.  Each loop
+ * runs with the values declared when it is called, in a graph capture too;
+ * a value that changes there ends the fusion of the loops on either side. */
 void op2_decl_const_char(int dim, char const *type, int size, char *data,
                          char const *name);
 

@@ -499,6 +499,13 @@ void op2_decl_const_char(int dim, char const *type, int size, char *data, char c
   c.dim = dim;
   c.size = size;
   c.bytes.assign(data, data + (size_t)dim * size);
+  // a capture launches loops after their call, with the constants declared by
+  // then: those already called keep the value they were called with
+  const auto old = rt().consts.find(name);
+  if (rt().capturing && old != rt().consts.end() &&
+      (old->second.type != c.type || old->second.dim != c.dim || old->second.size != c.size ||
+       old->second.bytes != c.bytes))
+    fusion_launch();
   rt().consts[name] = c;
   auto it = rt().const_targets.find(name);
   if (it != rt().const_targets.end()) {

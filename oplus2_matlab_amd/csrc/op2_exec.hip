@@ -3111,10 +3111,14 @@ void launch_stage(bool next_takes_res) {
 }
 }  // namespace
 
-void fusion_flush() {
+void fusion_launch() {
   launch_stage(false);
   flush_chain();
   release_held(nullptr);
+}
+
+void fusion_flush() {
+  fusion_launch();
   sync_shadows();
   flush_fold();
   zero_dats().clear();

@@ -274,7 +274,10 @@ void forget_plan_caches(const Plan *p);
 // and mark_end the stop node
 int mark_begin(int kind);
 void mark_end(int mark);
-// loop fusion during graph capture: launch, or forget, a held loop
+// loop fusion during graph capture: launch the loops called so far (a constant
+// they read is about to change), the same and leave every dat in its own
+// buffer, or forget the loops held
+void fusion_launch();
 void fusion_flush();
 void fusion_drop();
 // dats known to hold zeros: forgotten when work the runtime does not see
