@@ -87,7 +87,9 @@ struct CellTiles {
   int *d_list = nullptr;             // per tile: ring cells, then nodes outside its run
   unsigned *d_rec = nullptr;         // 4 words per finished cell
   double *partials[2] = {nullptr, nullptr};  // rms partials per stage and tile, as StageBufs'
-  std::vector<int> first_of_block;   // first tile of each plan block, and the end
+  // first tile of each plan block, and the end; -1: the block is the second of
+  // its tile's pair
+  std::vector<int> first_of_block;
   std::vector<std::pair<op_map, int *>> tile_off;  // first tile of each mesh, as StageBufs'
   int stages() const { return whole ? kMaxStages : depth; }  // most per launch
   int rings(int nstages) const { return std::min(nstages, kMaxRings) - 1; }  // index above

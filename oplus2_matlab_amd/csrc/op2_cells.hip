@@ -635,7 +635,7 @@ CellTilesHost build_cell_tiles(const Plan &p, op_map pcell, size_t real_bytes, b
       if ((first - base) % part == 0 && end - first == p.part_size && b + 1 < p.nblocks &&
           p.owned_off[b + 2] <= piece_end) {
         end = p.owned_off[b + 2];
-        t.first_of_block[++b] = t.ntiles() + 1;  // (no piece, so no mesh, starts there)
+        t.first_of_block[++b] = -1;
       }
     }
     todo.assign(1, {first, end});

@@ -2143,9 +2143,15 @@ void prepare_capture() {
       for (size_t m = t->tile_off.size(); t->d_rec && m < b->tile_off.size(); m++) {
         int *d = nullptr;
         if (b->tile_off[m].second && !t->whole) {
+          // (a mesh that starts inside a pair of blocks, as parts of one piece
+          // of the cells can: its tile would hold cells of two meshes)
           std::vector<int> first(b->tile_first[m]);
-          for (int &f : first) f = t->first_of_block[f];
-          d = to_device(first);
+          bool inside = false;
+          for (int &f : first) {
+            f = t->first_of_block[f];
+            inside |= f < 0;
+          }
+          if (!inside) d = to_device(first);
         }
         t->tile_off.emplace_back(b->tile_off[m].first, d);
       }
