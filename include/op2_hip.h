@@ -136,6 +136,12 @@ void op2_exit(void);
  * Returns 0 on success. */
 int op2_par_loop(char const *name, op_set set, int nargs, op_arg *args);
 
+/* op2_par_loop for bindings that report errors themselves (the error mode
+ * returns them): forgets the error recorded before, and returns -1 also where
+ * the loop ran although an error was recorded, as the argument checks at
+ * OP_diags > 0 do. */
+int op2_par_loop_checked(char const *name, op_set set, int nargs, op_arg *args);
+
 /* No counterpart in the reference: op2_par_loop for callers that cannot
  * allocate device memory (code under graph capture by the caller, tight
  * serving loops, harnesses that forbid hipMalloc).  Runs save_soln,

@@ -1187,4 +1187,10 @@ int op2_par_loop(char const *name, op_set set, int nargs, op_arg *args) {
   API_END(-1)
 }
 
+int op2_par_loop_checked(char const *name, op_set set, int nargs, op_arg *args) {
+  op2_clear_error();
+  const int rc = op2_par_loop(name, set, nargs, args);
+  return rc == 0 && !rt().last_error.empty() ? -1 : rc;
+}
+
 }  // extern "C"

@@ -111,6 +111,7 @@ SIGNATURES = {
                           C.POINTER(C.c_int)]),
     "op2_exit": (None, []),
     "op2_par_loop": (C.c_int, [C.c_char_p, _P, C.c_int, C.POINTER(OpArg)]),
+    "op2_par_loop_checked": (C.c_int, [C.c_char_p, _P, C.c_int, C.POINTER(OpArg)]),
     "op2_par_loop_noalloc": (C.c_int, [C.c_char_p, _P, C.c_int, C.POINTER(OpArg)]),
     "op2_set_error_mode": (C.c_int, [C.c_int]),
     "op2_last_error": (C.c_char_p, []),
@@ -351,7 +352,7 @@ def op_par_loop(kernel, name: str, set_: Set, *args: OpArg) -> None:
         arr = _arg_array(n).from_buffer_copy(b"".join(args))
     else:
         arr = _arg_array(n)(*args)  # (refuses what is no argument)
-    if lib().op2_par_loop(_b(name), set_._p, n, arr) != 0:
+    if lib().op2_par_loop_checked(_b(name), set_._p, n, arr) != 0:
         raise OP2Error(lib().op2_last_error().decode(errors="replace"))
 
 
