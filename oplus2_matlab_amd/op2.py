@@ -232,8 +232,6 @@ _arg_arrays = {}
 
 
 def _type_bytes(type_):
-    if type(type_) is not str:
-        return _b(type_)
     b = _types.get(type_)
     if b is None:
         b = _types[type_] = _b(type_)
