@@ -329,7 +329,7 @@ def op_arg_gbl(data: np.ndarray, dim: int, type_: str, acc: int) -> OpArg:
         raise OP2Error("op_arg_gbl needs a C-contiguous numpy array")
     want = _NP_TYPE.get(type_)
     t = type_ if (want is not None and data.dtype == want) else "error"
-    if data.nbytes and data.flags.writeable:
+    if t != "error" and data.nbytes and data.flags.writeable:
         address = C.addressof(C.c_char.from_buffer(data))  # (a third of ctypes.data's time)
     else:
         address = data.ctypes.data

@@ -28,3 +28,10 @@ def test_type_name_outlives_the_call(dat, name):
     others = [b"%06d" % i for i in range(1000)]  # (take the place of what was freed)
     assert [a.type for a in args] == [b"double"] * 2
     assert len(others) == 1000
+
+
+def test_array_of_no_type(dat):
+    """Refused by the loop, not by making the argument: a type the runtime
+    does not have is the argument type "error" (common/op_lib.h:184-190)."""
+    a = op2.op_arg_gbl(np.zeros(1, "datetime64[s]"), 1, "double", op2.OP_INC)
+    assert a.type == b"error" and a.data
