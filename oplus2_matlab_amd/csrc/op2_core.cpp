@@ -323,6 +323,7 @@ static void clear_all() {
   r.auto_renumber = false;
   r.set_segments.clear();
   r.map_internal.clear();
+  r.map_most.clear();
   checkpoint_reset();
   for (auto &o : r.online)
     for (auto &ev : o.second.events)
@@ -1088,7 +1089,7 @@ unsigned char const *op2_generic_owner_keeps(char const *name, op_set set, int n
   if (!p) {
     // a tile of `part` targets holds at most 16383 elements: loops that might
     // exceed that are left to the coloured plan
-    const op_map_core *m = nullptr;
+    op_map m = nullptr;
     std::vector<std::pair<op_map, int>> pairs;
     for (int a = 0; a < nargs; a++) {
       if (args[a].argtype != OP_ARG_DAT || !args[a].map) continue;
@@ -1100,11 +1101,16 @@ unsigned char const *op2_generic_owner_keeps(char const *name, op_set set, int n
       m = args[a].map;
     }
     if (!m || pairs.size() > 4) return nullptr;
-    const int *t = map_host((op_map)m);
-    std::vector<int> count(m->to->size, 0);
-    int most = 0;
-    for (size_t i = 0; i < (size_t)m->dim * set->size; i++) most = std::max(most, ++count[t[i]]);
-    if ((long long)most * part > 16383) return nullptr;
+    // (a loop so refused asks at every call: 4M entries take 5 ms to count)
+    auto most = rt().map_most.find(m);
+    if (most == rt().map_most.end()) {
+      const int *t = map_host(m);
+      std::vector<int> count(m->to->size, 0);
+      int n = 0;
+      for (size_t i = 0; i < (size_t)m->dim * m->from->size; i++) n = std::max(n, ++count[t[i]]);
+      most = rt().map_most.emplace(m, n).first;
+    }
+    if ((long long)most->second * part > 16383) return nullptr;
     p = get_plan(req);
   }
   if (!p->d_keeps) {

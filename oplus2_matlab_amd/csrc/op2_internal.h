@@ -251,6 +251,9 @@ struct Runtime {
   bool auto_renumber_default = false;  // op2_set_auto_renumber
   std::map<op_set, std::vector<int>> set_segments;
   std::map<op_map, std::vector<int>> map_internal;
+  // the most entries of a map that name one element (the same under any
+  // numbering), where it has been asked for (op2_generic_owner_keeps)
+  std::map<op_map, int> map_most;
   // generic loop path: loops and device constants registered by the
   // translation units that compile the user kernels
   std::map<std::string, op2_loop_fn> loops;
