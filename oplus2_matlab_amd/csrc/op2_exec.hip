@@ -2798,7 +2798,9 @@ void leave_fold(const Stage &st, StageBufs *sb, int par, const double *partials,
   if (f.nseg > 0 || f.n > 0) pending_fold() = PendingFold{true, f};
 }
 
-// Stages st[0 .. n) as one launch on cell tiles, the new q to q_dst.
+// Stages st[0 .. n) as one launch on cell tiles, the new q to q_dst.  kind: what
+// a timed launch of one stage runs (mark_begin counts it); -1: a group of a
+// march, which is not timed and counted there.
 template <typename T>
 void run_cells(const Stage *st, int n, const CellTiles *ct, char *q_dst, T *qold_out, int kind) {
   Runtime &r = rt();
@@ -2848,7 +2850,7 @@ void run_cells(const Stage *st, int n, const CellTiles *ct, char *q_dst, T *qold
       has_bres ? bres_idx<T>(st->bres.data(), (int)st->bres.size(), false) : BresIdx<T>{};
   const CarriedFold fold = take_fold(a.nfold);
   const int threads = std::max((ct->max_done[g] + kWave - 1) / kWave * kWave, kFixedBlock);
-  const int mark = n == 1 ? mark_begin(kind) : -1;
+  const int mark = kind >= 0 ? mark_begin(kind) : -1;
   const AirfoilConsts<T> k = airfoil_consts<T>();
   a.rcfl = near_reciprocal(k.cfl);
   launch_cells<T>(threads, a, bi, k, fold,
@@ -3041,7 +3043,7 @@ void run_march(std::vector<Stage> &c, const CellTiles *ct) {
     live_buf()[qold] = u.from == 0 ? own[0] : nullptr;
     const bool save = !c[u.first + u.n - 1].save.empty();
     const int to = 1 - u.from;
-    run_cells<T>(&c[u.first], u.n, ct, own[to], nullptr, 0);
+    run_cells<T>(&c[u.first], u.n, ct, own[to], nullptr, -1);
     r.capture_stages += u.n;
     live_buf()[qold] = (save ? to : u.from) == 0 ? own[0] : nullptr;
   }
