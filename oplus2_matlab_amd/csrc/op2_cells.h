@@ -49,11 +49,13 @@ constexpr int kCus = 256;
 // one stage a launch on single blocks.  us per iteration, one ring on single
 // blocks, two rings on single blocks, two rings on pairs:
 //   cells        FP64               FP32
-//   45k     11.8  10.3  12.5   10.7   8.8   9.8
-//   180k    18.5  17.2  19.0   13.9  12.5  13.8
-//   361k    29.5  29.7  27.2   19.8  21.4  19.1
-//   721k    46.6  49.1  46.7   31.1  36.9  34.0
-//   2.88M   162.8 176.5 149.5  84.2  122.8 99.3
+//   45k     11.9  10.1  12.4   10.8   8.4   9.5
+//   180k    18.0  16.2  18.4   13.8  11.9  12.9
+//   361k    28.7  29.3  26.2   19.0  21.0  18.0
+//   721k    44.7  48.9  46.8   29.6  36.4  33.2
+//   2.88M   165.6 178.3 148.4  82.3  123.5 98.0
+// (The rule is not the best everywhere: at 361k FP32 pairs are 5% faster, at
+// 721k FP64 single blocks are.)
 struct CellForm {
   int rings;
   bool wide;
@@ -147,9 +149,11 @@ inline size_t cells_lds(size_t real_bytes, int cap, int nodes) {
 // that they alternate between (three states, two adt, x and the records)
 // exceed 4/3 of the 256 MB last-level cache, a q kept there would be gone
 // before the next stage reads it, and takes the place of data that would
-// still be found.  Per iteration FP64 2.88M cells (409 MB) 187.6 us cached,
-// 176.0 past the caches; 2.0M (284 MB) 116.5 and 120.7; FP32 5.4M (421 MB)
-// 198.8 and 190.4, 3.9M (306 MB) 130.3 and 134.4.
+// still be found.  us per iteration, cached and past the caches: FP64 1.45M
+// cells (206 MB) 79.2 and 81.4, 2.0M (284 MB) 104.6 and 107.5, 2.88M (409 MB)
+// 155.8 and 148.7; FP32 2.88M (226 MB) 82.2 and 86.3, 3.9M (306 MB) 118.2 and
+// 113.8, 5.4M (421 MB) 176.5 and 170.8.  (FP64 changes over between 284 and
+// 409 MB; the FP32 form already between 226 and 306, by 4%.)
 inline bool cells_stream(size_t real_bytes, size_t cells, size_t nodes) {
   return (14 * real_bytes + 16) * cells + 2 * real_bytes * nodes > (size_t)256 * 1000000 / 3 * 4;
 }

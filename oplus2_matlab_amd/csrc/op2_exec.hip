@@ -21,10 +21,11 @@
 
 namespace op2 {
 
-// Threads per workgroup of the kernels whose size is fixed (the folds of
-// reduction partials and the copies of graph buffers).  Every other kernel
-// takes its workgroup size NT as a template parameter (128, 256 or 512: the
-// loop's block size), and the host code launching it passes the same NT.
+// Folds of reduction partials and copies of graph buffers run on kFixedBlock
+// threads, cell tiles on as many as they have cells to finish.  Every other
+// kernel takes its workgroup size NT as a template parameter (128, 256 or
+// 512: the loop's block size), and the host code launching it passes the same
+// NT.
 
 // ============================================================================
 // kernels
@@ -376,8 +377,9 @@ __device__ __forceinline__ op2_v4i position_ids(const int4 *__restrict__ ids,
   return __builtin_nontemporal_load((const op2_v4i *)(ids + pos));
 }
 
-// One edge of a gather tile: gathers, flux into LDS (component-major).  Each gather instruction takes the lower-numbered
-// node (cell) of every position, the next one the higher-numbered:
+// One edge of a gather tile: gathers, flux into LDS (component-major).  Each
+// gather instruction takes the lower-numbered node (cell) of every position,
+// the next one the higher-numbered:
 // positions follow their smaller cell, so neighbouring lanes then read
 // neighbouring records (fewer L1 lines per instruction than the map's slot
 // order, whose orientation is arbitrary).  The pairs are swapped back in
@@ -1316,11 +1318,11 @@ int part_of(const std::string &loop, int dflt) {
 }
 
 // Tiles of the fused stage kernels (op2_set_stage_config).  By default 256
-// cells on 256 threads whatever res_calc's own configuration: a stage tile
-// runs flux, update and adt_calc phases, and more, smaller workgroups per CU
-// overlap those phases better (2.88M cells: 256/256 beat res_calc's tuned
-// 512/512 by 5% in FP64 and 4% in the FP32 form; 128-cell tiles exceed the
-// side form of adt_calc).
+// cells on 256 threads whatever res_calc's own configuration: a stage of the
+// general kernel runs flux, update and adt_calc phases, and more, smaller
+// workgroups per CU overlap those phases better (2.88M cells: 256/256 beat
+// res_calc's tuned 512/512 by 5% in FP64 and 4% in the FP32 form).  Cell tiles
+// are cut from the same blocks.
 int stage_part_of(const std::string &loop) {
   const Runtime &r = rt();
   return r.stage_part < 0 ? part_of(loop, 256) : r.stage_part ? r.stage_part : 256;

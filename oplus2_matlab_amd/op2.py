@@ -566,7 +566,8 @@ def set_stage_config(part_size: int = 0, block_size: int = 0) -> None:
 
 
 # kinds of graph_kernel_times: the loops a stage kernel runs besides
-# res_calc and update, its res traffic, and the form of its adt_calc
+# res_calc and update, its res traffic, whether it runs on cell tiles with an
+# adt_calc (ADT_SIDES), and where it writes and reads qold
 KIND_BRES, KIND_SAVE, KIND_ADT, KIND_READS_RES, KIND_STORES_RES = 1, 2, 4, 8, 16
 KIND_ADT_SIDES, KIND_SAVE_IN_PLACE, KIND_QOLD_IS_Q = 32, 64, 128
 
