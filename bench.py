@@ -13,13 +13,18 @@ fuses loops that can share a pass: update with the next iteration's
 save_soln and each update or save_soln with the adt_calc that follows
 (--no-fusion captures the loops one kernel each).
 
-roofline: the stage kernel launched for one Runge-Kutta stage (res_calc,
-bres_calc, update and the next save_soln and adt_calc).  achieved =
-algorithmic bytes of its launches (stage_bytes: each map and dat it touches
-once per direction) divided by their device time, from event-record nodes that
-the runtime places around every 7th stage of graphs captured for this beside
-the timed ones (op2_set_graph_kernel_timing; in the timed graphs the stages of
-an iteration may share a launch).
+roofline: an iteration of the timed graphs (cell tiles: res_calc, bres_calc,
+update and the next save_soln and adt_calc of each stage in one kernel, the
+stages of an iteration in one launch or in one each).  achieved = the bytes
+that an iteration cannot do without (iteration_bytes) divided by the timed
+replays' wall time per iteration, so launches, gaps and the graph's ends count
+as time and the reads of a second launch do not count as bytes; traffic = the
+HBM bytes that the committed counter summary measured per iteration.  Under
+stage_alone: the stage kernel launched for one stage, in graphs of its own,
+whose every 7th stage the runtime brackets with event-record nodes
+(op2_set_graph_kernel_timing); bytes by cell_stage_bytes.  A mesh without cell
+tiles runs the general stage kernel, one launch per stage: roofline is then
+that kernel's, from the event-record nodes (stage_bytes).
 res_calc_roofline: the same for res_calc alone (76 B/edge FP64), from HIP
 events the runtime records on its stream around every loop call of an eager
 timed region; each of those calls follows an update, so the runtime takes
@@ -110,8 +115,8 @@ def parse():
                     help="iterations per captured graph (at most the step count; a second "
                          "graph runs the remainder)")
     ap.add_argument("--no-kernel-marks", dest="kernel_marks", action="store_false",
-                    help="capture the timed graphs without the event-record nodes that time "
-                         "their stage kernels")
+                    help="skip the graphs that time single stage kernels (roofline is then "
+                         "res_calc's)")
     return ap.parse_args()
 
 
@@ -265,12 +270,53 @@ def stage_bytes(mesh, kind, size):
     return b
 
 
+def cell_stage_bytes(mesh, kind, size):
+    """stage_bytes of a stage on cell tiles: in place of the edge maps and
+    pcell (or recipes) it reads one 16-byte record per cell."""
+    from oplus2_matlab_amd import op2
+
+    plain = kind & ~(op2.KIND_ADT | op2.KIND_ADT_SIDES)
+    return stage_bytes(mesh, plain, size) - 16 * mesh.nedge + 16 * mesh.ncell
+
+
+def iteration_bytes(mesh, size):
+    """Bytes an iteration on cell tiles cannot do without: q, adt, x and the
+    records (16 B per cell) read once, the new q and adt written once, 16 B
+    per boundary edge (its qold is the q it starts from)."""
+    return (10 * size + 16) * mesh.ncell + 2 * size * mesh.nnode + 16 * mesh.nbedge
+
+
+CELLS_PROFILE = os.path.join("profiles", "airfoil_cells_kernel_stats.md")
+
+
+def cells_traffic(ni, nj, size):
+    """Measured HBM bytes per iteration of the cell kernel's launches from the
+    committed counter summary (2400x1200, default tiles); else None."""
+    path = os.path.join(ROOT, CELLS_PROFILE)
+    if (ni, nj) != (2400, 1200) or not os.path.exists(path):
+        return None
+    form, table = {8: "FP64", 4: "FP32 form"}[size], False
+    for line in open(path):
+        table = table or line.startswith("HBM traffic per iteration")
+        f = [c.strip() for c in line.split("|")]
+        if table and len(f) > 6 and f[1] == form:
+            return float(f[6]) * 1e6
+    return None
+
+
+def on_cell_tiles(stages):
+    from oplus2_matlab_amd import op2
+
+    return any(kind & op2.KIND_ADT_SIDES for kind, _ in stages)
+
+
 def stage_roofline(mesh, stages, size):
-    """Stage kernels of the timed graphs: algorithmic bytes and device time
+    """Stage kernels launched one by one: algorithmic bytes and device time
     summed over the bracketed launches of each graph's last replay."""
     if not stages:
         return None
-    nbytes = sum(stage_bytes(mesh, kind, size) for kind, _ in stages)
+    of = cell_stage_bytes if on_cell_tiles(stages) else stage_bytes
+    nbytes = sum(of(mesh, kind, size) for kind, _ in stages)
     secs = sum(ms for _, ms in stages) * 1e-3
     by_kind = {}
     for kind, ms in stages:
@@ -278,7 +324,7 @@ def stage_roofline(mesh, stages, size):
     return {"launches": len(stages), "bytes_per_launch": nbytes / len(stages),
             "us_per_launch": 1e6 * secs / len(stages), "GBs": nbytes / secs / 1e9,
             "by_kind": {str(kd): {"launches": len(v), "us_per_launch": 1e3 * sum(v) / len(v),
-                                  "bytes_per_launch": stage_bytes(mesh, kd, size)}
+                                  "bytes_per_launch": of(mesh, kd, size)}
                         for kd, v in sorted(by_kind.items())}}
 
 
@@ -470,13 +516,24 @@ def main():
     stage = stage_roofline(mesh, r64["stages"], 8)
     stage_cfg = dict(res_cfg or {}) if st_part < 0 else \
         {"part_size": st_part or 256, "block_size": (st_block or 256) if st_part else 256}
-    if stage:
-        # (the committed counter summary's stage rows are those of the general
-        # stage kernel, which this mesh does not run)
+    if stage and on_cell_tiles(r64["stages"]):
+        needed = iteration_bytes(mesh, 8)
+        gbs = needed / r64["ms_per_step"] / 1e6
+        default_tiles = (stage_cfg.get("part_size"), stage_cfg.get("block_size")) == (256, 256)
+        traffic = cells_traffic(ni, nj, 8) if profiled and default_tiles else None
+        roofline = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": gbs / HBM_PEAK_GBS, "traffic": traffic,
+                    "traffic_source": CELLS_PROFILE if traffic else None,
+                    "kernel": "k_cells (the stages of an iteration: res_calc, bres_calc, update, "
+                              "save_soln, adt_calc) in the timed graphs, per iteration",
+                    "bytes_per_iteration": needed,
+                    "us_per_iteration": 1e3 * r64["ms_per_step"],
+                    "stage_alone": dict(stage, frac=stage["GBs"] / HBM_PEAK_GBS)}
+    elif stage:
         roofline = {"bound": "hbm", "achieved": stage["GBs"], "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": stage["GBs"] / HBM_PEAK_GBS, "traffic": None,
-                    "kernel": "k_cells (one Runge-Kutta stage: res_calc, bres_calc, update, "
-                              "save_soln, adt_calc), launched for one stage",
+                    "kernel": "k_stage (one Runge-Kutta stage: res_calc, bres_calc, update, "
+                              "save_soln, adt_calc)",
                     "bytes_per_launch": stage["bytes_per_launch"],
                     "us_per_launch": stage["us_per_launch"], "launches": stage["launches"],
                     "by_kind": stage["by_kind"]}
