@@ -2581,6 +2581,7 @@ bool overwrites_held_res(const char *name, Loop l, op_set set, int nargs, op_arg
   if (!h.active || h.adt_args.empty() || l != Loop::kResCalc) return false;
   if (h.l != Loop::kUpdate && h.l != Loop::kUpdateBatch) return false;
   if (a[6].dat != h.args[2].dat || a[6].map->to != h.set) return false;
+  if (exposed_dats().count(a[6].dat)) return false;  // (res_calc will read it)
   auto ot = rt().online.find(name);
   if (ot != rt().online.end() && !ot->second.done) return false;
   const int strategy = strategy_of(name);
@@ -3216,7 +3217,8 @@ int run_loop(const char *name, op_set set, int nargs, op_arg *args) {
   if (fuse) {
     if (stage_takes(l, rb, set, nargs, args)) return 0;
     Plan *sp = starts_stage(name, l, rb, set, nargs, args);
-    launch_stage(sp && stage().res.size() > 6 && stage().res[6].dat == args[6].dat);
+    launch_stage(sp && stage().res.size() > 6 && stage().res[6].dat == args[6].dat &&
+                 !exposed_dats().count(args[6].dat));
     if (sp) {
       // a stage reads q and adt where they are (the previous stage's
       // outputs); anything held from before is launched first
