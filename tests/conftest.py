@@ -15,6 +15,12 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: takes more than ~20 s on the CPU")
 
 
+def pytest_collection_modifyitems(items):
+    # the programs built from the reference's sources come last: where those
+    # are absent, a run that ends at the first failure has run the rest
+    items.sort(key=lambda i: i.path.name == "test_gpu_dropin.py")
+
+
 @pytest.fixture(scope="session")
 def golden_dir():
     return GOLDEN
